@@ -482,11 +482,22 @@ __global__ __launch_bounds__(1024) void tri_tear_kernel(DcWork w, const double *
   }
 }
 
+// Whether an earlier launch failed, the same answer for every thread of the workgroup. Other
+// workgroups of this launch may clear the status at any time: if each wave read it for itself,
+// some could leave and the others go on past the barriers with LDS entries nobody wrote, which
+// index memory below. (The kernels without barriers let each thread read it.)
+__device__ __forceinline__ bool failed(const DcWork &w) {
+  __shared__ int status;
+  if (threadIdx.x == 0) status = w.info[1];
+  __syncthreads();
+  return status == 0;
+}
+
 // One leaf per workgroup, by dc_eig.hpp's tridiagonal solver.
 __global__ __launch_bounds__(kLeafThreads) void tri_leaf_kernel(DcWork w, double *__restrict__ Q,
                                                                 double *__restrict__ Q2, double *__restrict__ U) {
   __shared__ dc::DcShared sh;
-  if (w.info[1] == 0) return;
+  if (failed(w)) return;
   const int b = blockIdx.x * w.leaf, s = w.leaf, t = threadIdx.x;
   const int64_t P = w.Pp, o = b * (P + 1);
   for (int i = t; i < s; i += kLeafThreads) {
@@ -520,7 +531,7 @@ __global__ __launch_bounds__(1024) void tri_deflate_kernel(DcWork w, int n, int 
   __shared__ double red[2][16];
   __shared__ int cnt[1024];
   __shared__ int bad, nrot;
-  if (w.info[1] == 0) return;
+  if (failed(w)) return;
   const int m = blockIdx.x, b = m * n, s = n / 2, t = threadIdx.x;
   const int64_t P = w.Pp;
   const double *lam = w.lam[cur] + b;
@@ -749,7 +760,7 @@ __global__ __launch_bounds__(256) void tri_couple_kernel(DcWork w, int n, int ni
 __global__ __launch_bounds__(256) void tri_vec_kernel(DcWork w, int n, double *__restrict__ U) {
   extern __shared__ double u[];
   __shared__ double red[4];
-  if (w.info[1] == 0) return;
+  if (failed(w)) return;
   const int a = blockIdx.x, m = a / n, b = m * n, x = a - b, K = w.mK[m], t = threadIdx.x;
   const int64_t P = w.Pp;
   for (int i = t; i < n; i += 256) u[i] = 0.0;

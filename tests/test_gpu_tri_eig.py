@@ -69,3 +69,19 @@ def test_tri_eig_spectra(ctx, rng, cplx, p, kind):
     else:
         M = np.zeros((p, p), dtype=complex if cplx else float)
     check(np.asfortranarray(M), kind in ("graded", "repeated", "diagonal") and kind != "graded")
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("p", [160, 530])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_tri_eig_failure_is_reported(ctx, rng, cplx, p, value):
+    """A non-finite entry: the solver reports failure, the paths behind it refuse the matrix too,
+    the call ends with a status, and the next call on the same workspaces is right."""
+    from tnhip import Tensor, TnhError, ops as T
+
+    M = randn(rng, (p, p + 3), cplx)
+    M[3, 7] = value
+    with pytest.raises(TnhError) as e:
+        T.svd_trunc(Tensor.from_numpy(M), 0.0, 0, 1)
+    assert e.value.status in (-5, -6)
+    check(randn(rng, (p, p + 3), cplx), True)
