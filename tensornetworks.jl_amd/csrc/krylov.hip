@@ -35,8 +35,8 @@ __device__ __forceinline__ double wave_tree(double v) {
   return dc::xor_sum<1>(dc::xor_sum<2>(dc::xor_sum<4>(dc::xor_sum<8>(dc::xor_sum<16>(dc::xor_sum<32>(v))))));
 }
 
-// s + p with the product rounded before it is added (no contraction), as the separate kernels
-// of a Krylov step are compiled
+// s + a b with the product rounded before it is added. Every form of a real Krylov step sums
+// with it, so that the forms give the same bits whatever the compiler would contract.
 __device__ __forceinline__ double add_rounded(double s, double a, double b) {
 #pragma clang fp contract(off)
   const double p = a * b;
@@ -99,8 +99,12 @@ __global__ __launch_bounds__(1024) void mdot1_kernel(const double *__restrict__ 
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      sr += vr[u] * wr[u] + vi[u] * wi[u];
-      si += vr[u] * wi[u] - vi[u] * wr[u];
+      if (cplx) {
+        sr += vr[u] * wr[u] + vi[u] * wi[u];
+        si += vr[u] * wi[u] - vi[u] * wr[u];
+      } else {
+        sr = add_rounded(sr, vr[u], wr[u]);
+      }
     }
   }
   __shared__ double red[2][16];
@@ -162,7 +166,7 @@ __global__ __launch_bounds__(256) void vsub_dev_kernel(double *__restrict__ w,
         ar -= cr[i] * vr - ci[i] * vi;
         ai -= cr[i] * vi + ci[i] * vr;
       } else {
-        ar -= cr[i] * vr;
+        ar = add_rounded(ar, -cr[i], vr);
       }
     }
     w[k] = ar;
@@ -187,8 +191,8 @@ __global__ __launch_bounds__(256) void normalize_copy_kernel(double *__restrict_
 // V[nv] = w / |w|; hj receives the coefficients and |w|^2 as the separate kernels would leave
 // them. Bound by the chain of one reduction per vector and pass. The sums run in
 // mdot1_kernel's order (threads stride 1024, then the wave tree, then the waves in turn) with
-// products rounded where the separate kernels round them, so a step gives the same bits as
-// they do: in a sweep of small splits the last bits of a vector move the energies.
+// rounded products (add_rounded), so a step gives the same bits as the separate kernels: in a
+// sweep of small splits the last bits of a vector move the energies.
 // Per step, this / separate launches, us: n 1024, nv 1 / 4 / 8: 4.9 / 10.1 / 16.9 vs 15.1 /
 // 16.0 / 17.1; n 4096, nv 4: 17.4 vs 17.8; n 8192, nv 2 / 4: 16.1 / 27.7 vs 19.6 / 20.2; n
 // 16384, nv 1: 16.5 vs 25.0. Hence the lines nv <= 8 and nv n <= 16384. (A complex form took

@@ -39,3 +39,34 @@ def test_lanczos_forms(ctx, rng, chi, kdim, cplx):
     assert abs(e - e0) <= 1e-11 * max(1.0, abs(e0))
     assert abs(abs(np.vdot(v, y)) - 1) <= 1e-9
     assert abs(np.linalg.norm(v) - 1) <= 1e-12
+
+
+@pytest.mark.parametrize("cr,kdim", [(32, 3), (16, 8), (31, 4)])
+def test_step_forms_same_bits(ctx, rng, cr, kdim):
+    """The one-launch step and the separate kernels on one input give the same bits. The input
+    padded with zeros to 16384 entries takes the separate kernels from the second vector on (all
+    its sums meet the same entries in the same order, then zeros). The operator is diagonal with
+    powers of two, so that the products before a step are exact at either size."""
+    from tnhip import Tensor, ops as T
+
+    cl, wide = 32, 128  # 32 x 2 x 2 x 128 = 16384
+
+    def diag(n, seed):
+        g = np.random.default_rng(seed)
+        a = np.zeros((n, 1, n))
+        a[np.arange(n), 0, np.arange(n)] = g.choice([-1.0, 1.0], n) * 2.0 ** g.integers(-3, 3, n)
+        return np.asfortranarray(a)
+
+    W = np.zeros((1, 2, 2, 1))
+    W[0, :, :, 0] = np.diag([1.0, 0.5])
+    R = diag(wide, 1)
+    x = np.zeros((cl, 2, 2, wide), order="F")
+    x[..., :cr] = rng.standard_normal((cl, 2, 2, cr))
+    got = []
+    for c in (cr, wide):
+        th = Tensor.from_numpy(np.asfortranarray(x[..., :c]))
+        e, nmv = T.eigsolve_ground(Tensor.from_numpy(diag(cl, 0)), Tensor.from_numpy(W), Tensor.from_numpy(W),
+                                   Tensor.from_numpy(np.asfortranarray(R[:c, :, :c])), th, krylovdim=kdim, maxiter=2)
+        got.append((e, nmv, th.numpy()))
+    assert got[0][:2] == got[1][:2] and got[0][1] >= 2 * kdim - 1
+    assert np.array_equal(got[0][2], got[1][2][..., :cr]) and not got[1][2][..., cr:].any()
