@@ -1,4 +1,4 @@
-"""Large products whose k range is split (csrc/gemm.hip, ksplit_wanted) against numpy: k a
+"""Large products whose k range is split (csrc/gemm_split.hpp, ksplit_wanted) against numpy: k a
 multiple of nothing, odd sides and leading dimensions, alpha and beta, every mode, and a
 product just below the k from which a split is considered.
 
@@ -10,10 +10,17 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+SLICES = {  # M, N, K: the slices of each mode on 256 CUs (tests/test_gemm_split_host.py)
+    (2804, 593, 2965): {"f64": 3, "f32": 4, "bf16x3": 4},
+    (2048, 700, 2049): {"f64": 2, "f32": 4, "bf16x3": 4},
+    (1100, 1283, 2500): {"f64": 2, "f32": 4, "bf16x3": 4},
+    (1100, 1283, 2047): {"f64": 1, "f32": 1, "bf16x3": 1},
+}
+
 
 @pytest.mark.parametrize("prec", ["f64", "f32", "bf16x3"])
 @pytest.mark.parametrize("ops", ["NN", "NT", "TN"])
-@pytest.mark.parametrize("mnk", [(2804, 593, 2965), (2048, 700, 2049), (1100, 1283, 2500), (1100, 1283, 2047)])
+@pytest.mark.parametrize("mnk", SLICES)
 def test_split_product(ctx, rng, mnk, ops, prec):
     from tnhip import Tensor, ops as T
 

@@ -1,7 +1,7 @@
 """The 256 x 256 tiles (csrc/gemm_wide.hip, csrc/gemm_wide_bf16.hip) against numpy: sides one vector into a tile or
 short of it, k below, at and above whole k-steps, strides, alpha and beta, both output types, k
 slices; and, FP32 unsplit, bit for bit against the other tiles, which a product with an odd
-leading dimension takes.
+leading dimension takes. tests/test_gemm_split_host.py holds the sizes to the kernels they are for.
 
 Tolerance, of the result (zero-mean operands): FP32 sums 2e-6 sqrt(K / 64), split-BF16x3 3e-5."""
 import numpy as np
@@ -9,16 +9,25 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [  # M, N, K: at least 0.9 of whole rounds of tiles on 256 CUs
+SIZES = [  # M, N, K of one slice, at least 0.9 of whole rounds of tiles on 256 CUs
     (4096, 4096, 256), (4092, 3844, 260), (3844, 4096, 287), (4096, 4088, 317),
-    (2048, 4096, 4100), (3076, 4084, 2049),  # split
 ]
+# products in slices of k, with the kernel and the slices of each mode; the last two are on the
+# other side of the line (the kernel of one 128 x 128 tile a workgroup)
+SLICED = {
+    (752, 6732, 8064): {"f32": ("wide", 3), "bf16x3": ("wide", 3)},
+    (756, 6732, 8067): {"f32": ("wide", 3), "bf16x3": ("wide", 3)},
+    (5116, 1276, 5132): {"f32": ("wide", 5), "bf16x3": ("tiles", 1)},
+    (2048, 4096, 4100): {"f32": ("tiles", 1), "bf16x3": ("tiles", 1)},
+    (3076, 4084, 2049): {"f32": ("tiles", 3), "bf16x3": ("wide", 1)},
+}
+SAME_BITS = [(4092, 3844, 300)]
 
 
 @pytest.mark.parametrize("prec", ["f32", "bf16x3"])
 @pytest.mark.parametrize("out", ["f32", "f64"])
 @pytest.mark.parametrize("ops", ["NN", "NT", "TN"])
-@pytest.mark.parametrize("mnk", SIZES)
+@pytest.mark.parametrize("mnk", SIZES + list(SLICED))
 def test_wide_product(ctx, rng, mnk, ops, out, prec):
     from tnhip import Tensor, ops as T
 
@@ -47,7 +56,7 @@ def test_wide_product(ctx, rng, mnk, ops, out, prec):
 def test_same_bits_as_other_tiles(ctx, rng, ops):
     from tnhip import Tensor, ops as T
 
-    M, N, K = 4092, 3844, 300
+    M, N, K = SAME_BITS[0]
     A = rng.standard_normal((K, M) if ops[0] == "T" else (M, K), dtype=np.float32)
     B = rng.standard_normal((N, K) if ops[1] == "T" else (K, N), dtype=np.float32)
     dA, dB = (Tensor.from_numpy(x, np.float32, ctx=ctx) for x in (A, B))
