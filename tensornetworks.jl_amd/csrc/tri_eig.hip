@@ -1,5 +1,4 @@
-// Eigen-decomposition of a Hermitian matrix of side 9 .. kTriMax(Cplx) spread over the whole
-// GPU: Householder reduction to a real symmetric tridiagonal matrix, divide and conquer with
+// Eigen-decomposition of a Hermitian matrix (sides: tri_eig.hpp) spread over the whole GPU: Householder reduction to a real symmetric tridiagonal matrix, divide and conquer with
 // one launch per phase and level, back-transformation by blocked reflectors on the matrix
 // cores. It replaces two solvers for the Gram matrices of cold splits: the one-workgroup
 // reduction (whose p steps stream the matrix through one CU: 25 ms at p = 512) and, above
@@ -398,20 +397,16 @@ template <bool CPLX>
 void launch_tail(hipStream_t st, const double *A, int64_t im, int p, int k0, const double *y, double *V, double *dd,
                  double *ee, double *taus) {
   const int m = p - k0;
-  if (m <= 32)
-    run_tail<CPLX, 256, 2, 2>(st, A, im, p, k0, y, V, dd, ee, taus);
-  else if (m <= 64)
-    run_tail<CPLX, 256, 4, 4>(st, A, im, p, k0, y, V, dd, ee, taus);
-  else if (m <= 96)
-    run_tail<CPLX, 256, 6, 6>(st, A, im, p, k0, y, V, dd, ee, taus);
-  else if (m <= 128)
-    run_tail<CPLX, 512, 4, 8>(st, A, im, p, k0, y, V, dd, ee, taus);
-  else if constexpr (!CPLX) {
-    if (m <= 160)
-      run_tail<false, 512, 5, 10>(st, A, im, p, k0, y, V, dd, ee, taus);
-    else
-      run_tail<false, 512, 6, 12>(st, A, im, p, k0, y, V, dd, ee, taus);
+  if constexpr (CPLX) {
+    if (m <= 32) return run_tail<true, 256, 2, 2>(st, A, im, p, k0, y, V, dd, ee, taus);
+    if (m <= 64) return run_tail<true, 256, 4, 4>(st, A, im, p, k0, y, V, dd, ee, taus);
+    if (m <= 96) return run_tail<true, 256, 6, 6>(st, A, im, p, k0, y, V, dd, ee, taus);
+  } else {
+    static_assert(kTriMinReal > 96, "smaller real tails are not instantiated");
+    if (m > 160) return run_tail<false, 512, 6, 12>(st, A, im, p, k0, y, V, dd, ee, taus);
+    if (m > 128) return run_tail<false, 512, 5, 10>(st, A, im, p, k0, y, V, dd, ee, taus);
   }
+  run_tail<CPLX, 512, 4, 8>(st, A, im, p, k0, y, V, dd, ee, taus);
 }
 
 // ------------------------------------------------------------------ divide and conquer
@@ -938,9 +933,9 @@ void launch_back(tnh_ctx *ctx, const double *V, int p, const double *taus, doubl
   const dim3 grid(unsigned((k + 3) / 4)), block(256);
   const int64_t im = int64_t(p) * p, imX = int64_t(p) * k;
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, ctx->stream, V, p, im, taus, X, imX, k); };
-  if (p <= 64)
-    go(tri_back_kernel<CPLX, 1>);
-  else if (p <= 128)
+  if constexpr (CPLX)
+    if (p <= 64) return go(tri_back_kernel<true, 1>);
+  if (p <= 128)
     go(tri_back_kernel<CPLX, 2>);
   else if (p <= 192)
     go(tri_back_kernel<CPLX, 3>);
@@ -996,7 +991,8 @@ T *carve(char *&at, int64_t n) {
 }  // namespace
 
 void tri_eig_solve(tnh_ctx *ctx, double *G, int p, bool cplx, double *dout) {
-  TNH_REQUIRE(p >= 2 && p <= (cplx ? kTriMaxCplx : kTriMaxReal), TNH_ERR_ARG, "tri_eig: side out of range");
+  TNH_REQUIRE(p >= (cplx ? kTriMinCplx : kTriMinReal) && p <= (cplx ? kTriMaxCplx : kTriMaxReal), TNH_ERR_ARG,
+              "tri_eig: side out of range");
   const int64_t pp = int64_t(p) * p;
   const int PL = cplx ? 2 : 1;
   const Leaves lv = leaves_of(p);

@@ -85,3 +85,24 @@ def test_tri_eig_failure_is_reported(ctx, rng, cplx, p, value):
         T.svd_trunc(Tensor.from_numpy(M), 0.0, 0, 1)
     assert e.value.status in (-5, -6)
     check(randn(rng, (p, p + 3), cplx), True)
+
+
+@pytest.mark.parametrize("cplx,p", [(True, 1850), (True, 3072), (False, 6144)])
+def test_tri_eig_largest_sides(ctx, rng, cplx, p):
+    """The complex column step in one 1024-thread workgroup a CU (sides above 1800), and the
+    largest sides of either type, where the column step's vectors fill LDS. M = H1 H2 diag(s) H3
+    H4 with Householder reflections H, so its singular values are known."""
+    from tnhip import Tensor, ops as T
+
+    s = 2.0 - np.arange(p) / p
+    M = np.diag(s).astype(complex if cplx else float)
+    for _ in range(2):
+        v, w = randn(rng, (p, 1), cplx), randn(rng, (p, 1), cplx)
+        M -= v @ ((2.0 / np.linalg.norm(v) ** 2) * (v.conj().T @ M))
+        M -= (M @ w) @ ((2.0 / np.linalg.norm(w) ** 2) * w.conj().T)
+    U, S, Vt, _, fb = T.svd_trunc(Tensor.from_numpy(np.asfortranarray(M)), 0.0, 0, 1)
+    assert not fb
+    u, got, vt = U.numpy(), S.numpy(), Vt.numpy()
+    assert np.abs(got ** 2 - s ** 2).max() <= 1e-13 * np.sqrt(p) * s[0] ** 2
+    assert np.abs(u.conj().T @ u - np.eye(p)).max() <= 1e-12
+    assert np.linalg.norm((u * got) @ vt - M) <= 1e-12 * np.linalg.norm(M)
