@@ -325,9 +325,10 @@ void small_contract(tnh_ctx *ctx, const Small &s) {
   if (ev) {
     const double planes_in = cin ? 2 : 1, planes_out = (cin || cw) ? 2 : 1;
     const double cmul = (cin && cw) ? 4 : ((cin || cw) ? 2 : 1);
-    ctx->prof_end("mix", ev, 2.0 * cmul * double(p.total) * s.I * s.J,
-                  double(p.total) * (s.I * planes_in * real_size(s.tin) +
-                                     s.J * planes_out * real_size(s.tout) * (s.beta != 0.0 ? 2 : 1)));
+    const double sites = double(s.na) * double(s.nb);
+    ctx->prof_end("mix", ev, 2.0 * cmul * sites * s.I * s.J,
+                  sites * (s.I * planes_in * real_size(s.tin) +
+                           s.J * planes_out * real_size(s.tout) * (s.beta != 0.0 ? 2 : 1)));
   }
 }
 

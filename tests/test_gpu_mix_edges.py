@@ -51,3 +51,31 @@ def test_mix_in_environments(ctx, rng, chi, D, cplx):
     right = T.env_right(Tensor.from_numpy(R), Tensor.from_numpy(A), Tensor.from_numpy(W)).numpy()
     ref = np.tensordot(np.tensordot(np.tensordot(A, R, (2, 2)), W, ((1, 3), (2, 3))), A.conj(), ((3, 1), (1, 2)))
     assert np.linalg.norm(right - ref.transpose(2, 1, 0)) <= 1e-13 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("prec,cplx", [("f64", False), ("f64", True), ("f32", False)])
+@pytest.mark.parametrize("chi", [(5, 7), (61, 34)])
+def test_mix_profiled_work(ctx, rng, chi, prec, cplx):
+    """The work the profile reports for one mixing pass of a matvec: cl cr (I + J) values moved
+    and cl cr I J multiply-adds (twice that with a complex input), whatever a thread takes."""
+    from tnhip import Tensor, ops as T
+
+    def rand(*s):
+        a = rng.standard_normal(s)
+        return np.asfortranarray(a + 1j * rng.standard_normal(s) if cplx else a)
+
+    (cl, cr), D, d = chi, 5, 2
+    dt = np.float32 if prec == "f32" else None
+    L, R = (Tensor.from_numpy(rand(c, D, c), dt, ctx=ctx) for c in chi)
+    W = Tensor.from_numpy(rng.standard_normal((D, d, d, D)), ctx=ctx)
+    x = Tensor.from_numpy(rand(cl, d, d, cr), ctx=ctx)
+    T.heff_apply(L, W, W, R, x, precision=prec)
+    ctx.profile_reset()
+    ctx.profile(True)
+    T.heff_apply(L, W, W, R, x, precision=prec)
+    got = ctx.profile_read("mix")
+    ctx.profile(False)
+    n, ij = cl * cr * (2 if cplx else 1), D * d * d
+    assert got["launches"] == 1
+    assert got["flops"] == 2 * n * ij * ij
+    assert got["bytes"] == n * 2 * ij * (4 if prec == "f32" else 8)
