@@ -33,18 +33,21 @@ struct SmallParams {
 
 // out[a, j, b] = sum_i in[a, i, b] * Wc[i, j]; a thread takes VA consecutive a of one b (a
 // fastest, so that a wave's loads and stores are contiguous runs) and jper of the J output
-// columns. EI is the compile-time I (0: any I up to MAXI), which unrolls the sum without a
-// test per term. Vectors need no alignment beyond the element's; the last one of a run is
-// read and written element by element when na is not a multiple of VA.
+// columns. NI is I rounded up to a multiple of four (WHOLE), with zeros for the terms past I, so
+// that the sum is unrolled and only its last three loads are conditional; above 32, and where
+// both factors are complex, it is the largest I instead, with a test per term. Vectors need no
+// alignment beyond the element's; the last one of a run is read and written element by element
+// when na is not a multiple of VA.
 //
-// Bound by HBM when large, by latency when small. Large: 16-byte accesses whatever na is
-// (FP64, na = 701, nb = 593, I = J = 20: 26 us, 5.1 TB/s, against 113 us with one element per
-// thread; FP32, 2048^2: 118 us, 5.7 TB/s, against 200 us with a test per term). Small: the launch splits
-// the J columns over blockIdx.y (the inputs of the others come from L2) until it has two waves
-// per SIMD, so a thread's chain is I loads and I multiply-adds per column it keeps, instead of
-// all I J (na = nb = 24, I = J = 12: 14 us with all columns in one thread, 4 us split). The sum over i is in
-// one order in every form.
-template <typename TI, typename TO, bool CIN, bool CW, int VA, int EI, int MAXI>
+// Bound by HBM when large, by latency when small. Large: 16-byte accesses whatever na is (FP64,
+// na = 701, nb = 593, I = J = 20: 26 us, 5.1 TB/s, against 113 us with one element per thread)
+// and no test per term (FP32, 2048^2, I = J = 20: 118 us, 5.7 TB/s, against 200; I = J = 28: 193
+// against 330; FP64, 500^2, 28: 34 against 62).
+// Small: the launch splits the J columns over blockIdx.y (the inputs of the others come from L2)
+// until it has two waves per SIMD, so a thread's chain is I loads and I multiply-adds per column
+// it keeps, instead of all I J (na = nb = 24, I = J = 12: 14 us with all columns in one thread,
+// 4 us split). The sum over i is in one order in every form.
+template <typename TI, typename TO, bool CIN, bool CW, int VA, int NI, bool WHOLE>
 __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
   using R = typename std::conditional<std::is_same<TI, double>::value ||
                                           std::is_same<TO, double>::value,
@@ -53,11 +56,13 @@ __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
   typedef TO VO __attribute__((ext_vector_type(VA), aligned(sizeof(TO))));
   extern __shared__ double wsm[];
   R *W = reinterpret_cast<R *>(wsm);
-  const int I = EI ? EI : p.I, j0 = blockIdx.y * p.jper, nj = min(p.J - j0, p.jper);
-  const int IJ = p.I * p.J, IN = I * nj;
+  const int I = p.I, j0 = blockIdx.y * p.jper, nj = min(p.J - j0, p.jper);
+  const int LD = WHOLE ? NI : I, IJ = I * p.J, IN = LD * nj;
   for (int e = threadIdx.x; e < IN; e += 256) {
-    W[e] = R(p.Wc[j0 * I + e]);
-    if constexpr (CW) W[IN + e] = R(p.Wc[IJ + j0 * I + e]);
+    const int i = WHOLE ? e % NI : 0, q = WHOLE ? (j0 + e / NI) * I + i : j0 * I + e;
+    const bool in = i < I;
+    W[e] = in ? R(p.Wc[q]) : R(0);
+    if constexpr (CW) W[IN + e] = in ? R(p.Wc[IJ + q]) : R(0);
   }
   __syncthreads();
 
@@ -87,30 +92,28 @@ __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
         if (u < left) q[u] = x[u];
     }
   };
-  constexpr int NI = EI ? EI : MAXI;
   R vr[NI][VA], vi[CIN ? NI : 1][VA];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    if (EI || i < I) {
-      VI x;
+    VI x = 0, y = 0;
+    if ((WHOLE && i + 3 < NI) || i < I) {
       load(in + p.offI[i], x);
+      if constexpr (CIN) load(in + p.in_im + p.offI[i], y);
+    }
 #pragma unroll
-      for (int u = 0; u < VA; ++u) vr[i][u] = R(x[u]);
-      if constexpr (CIN) {
-        load(in + p.in_im + p.offI[i], x);
-#pragma unroll
-        for (int u = 0; u < VA; ++u) vi[i][u] = R(x[u]);
-      }
+    for (int u = 0; u < VA; ++u) {
+      vr[i][u] = R(x[u]);
+      if constexpr (CIN) vi[i][u] = R(y[u]);
     }
   }
   for (int j = 0; j < nj; ++j) {
-    const R *wr = W + j * I, *wi = W + IN + j * I;
+    const R *wr = W + j * LD, *wi = W + IN + j * LD;
     R sr[VA], si[VA];
 #pragma unroll
     for (int u = 0; u < VA; ++u) sr[u] = si[u] = R(0);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      if (EI || i < I) {
+      if (WHOLE || i < I) {
         const R c = wr[i];
 #pragma unroll
         for (int u = 0; u < VA; ++u) sr[u] += vr[i][u] * c;
@@ -281,37 +284,40 @@ void small_contract(tnh_ctx *ctx, const Small &s) {
   const int64_t want = std::max<int64_t>(1, (2 * int64_t(ctx->cu_count) + blocks - 1) / blocks);
   p.jper = int((s.J + std::min<int64_t>(want, s.J) - 1) / std::min<int64_t>(want, s.J));
   const dim3 grid(unsigned(blocks), unsigned((s.J + p.jper - 1) / p.jper));
-  const size_t shm = size_t(s.I) * p.jper * (cw ? 2 : 1) * ((i64 || o64) ? 8 : 4);
+  const bool whole = s.I <= 32 && !(cin && cw);
+  const size_t shm = size_t(whole ? (s.I + 3) / 4 * 4 : s.I) * p.jper * (cw ? 2 : 1) * ((i64 || o64) ? 8 : 4);
   hipEvent_t ev = ctx->prof_begin();
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), shm, ctx->stream, p); };
   auto typed = [&](auto ti, auto to) {
     using TI = decltype(ti);
     using TO = decltype(to);
     constexpr int VA = (sizeof(TI) == 8 || sizeof(TO) == 8) ? 2 : 4;
-    if (cin && cw) {
-      s.I <= 16 ? go(mix_kernel<TI, TO, true, true, 1, 0, 16>) : go(mix_kernel<TI, TO, true, true, 1, 0, kMaxIJ>);
-    } else if (cin) {
-      switch (s.I) {  // d D and d^2 D of the usual chains: no test per term
-        case 6: return go(mix_kernel<TI, TO, true, false, 1, 6, 6>);
-        case 10: return go(mix_kernel<TI, TO, true, false, 1, 10, 10>);
-        case 12: return go(mix_kernel<TI, TO, true, false, 1, 12, 12>);
-        case 20: return go(mix_kernel<TI, TO, true, false, 1, 20, 20>);
+    auto rounded = [&](auto ci, auto cc, auto va) {
+      constexpr bool CI = decltype(ci)::value, CC = decltype(cc)::value;
+      constexpr int V = decltype(va)::value;
+      switch ((s.I + 3) / 4) {
+        case 0:
+        case 1: return go(mix_kernel<TI, TO, CI, CC, V, 4, true>);
+        case 2: return go(mix_kernel<TI, TO, CI, CC, V, 8, true>);
+        case 3: return go(mix_kernel<TI, TO, CI, CC, V, 12, true>);
+        case 4: return go(mix_kernel<TI, TO, CI, CC, V, 16, true>);
+        case 5: return go(mix_kernel<TI, TO, CI, CC, V, 20, true>);
+        case 6: return go(mix_kernel<TI, TO, CI, CC, V, 24, true>);
+        case 7: return go(mix_kernel<TI, TO, CI, CC, V, 28, true>);
+        case 8: return go(mix_kernel<TI, TO, CI, CC, V, 32, true>);
       }
-      s.I <= 32 ? go(mix_kernel<TI, TO, true, false, 1, 0, 32>) : go(mix_kernel<TI, TO, true, false, 1, 0, kMaxIJ>);
-    } else if (s.I > 32) {
-      cw ? go(mix_kernel<TI, TO, false, true, 1, 0, kMaxIJ>) : go(mix_kernel<TI, TO, false, false, 1, 0, kMaxIJ>);
-    } else if (cw) {
-      go(mix_kernel<TI, TO, false, true, VA, 0, 32>);
-    } else {
-      switch (s.I) {
-        case 6: return go(mix_kernel<TI, TO, false, false, VA, 6, 6>);
-        case 10: return go(mix_kernel<TI, TO, false, false, VA, 10, 10>);
-        case 12: return go(mix_kernel<TI, TO, false, false, VA, 12, 12>);
-        case 20: return go(mix_kernel<TI, TO, false, false, VA, 20, 20>);
-        case 32: return go(mix_kernel<TI, TO, false, false, VA, 32, 32>);
-      }
-      go(mix_kernel<TI, TO, false, false, VA, 0, 32>);
-    }
+      go(mix_kernel<TI, TO, CI, CC, 1, kMaxIJ, false>);
+    };
+    using one = std::integral_constant<int, 1>;
+    using vec = std::integral_constant<int, VA>;
+    if (cin && cw)
+      s.I <= 16 ? go(mix_kernel<TI, TO, true, true, 1, 16, false>) : go(mix_kernel<TI, TO, true, true, 1, kMaxIJ, false>);
+    else if (cin)
+      rounded(std::true_type(), std::false_type(), one());
+    else if (cw)
+      rounded(std::false_type(), std::true_type(), vec());
+    else
+      rounded(std::false_type(), std::false_type(), vec());
   };
   if (i64 && o64)
     typed(double(), double());

@@ -53,6 +53,26 @@ def test_mix_in_environments(ctx, rng, chi, D, cplx):
     assert np.linalg.norm(right - ref.transpose(2, 1, 0)) <= 1e-13 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("D,d", [(1, 2), (1, 3), (2, 3), (3, 3), (7, 2)])
+def test_mix_term_counts(ctx, rng, D, d, cplx):
+    """Term counts d^2 D of every remainder modulo four (4, 9, 18, 27, 28), with a value of 1e300
+    in the last term."""
+    from oracle.projmps import product_optimal
+    from tnhip import Tensor, ops as T
+
+    def rand(*s):
+        a = rng.standard_normal(s)
+        return np.asfortranarray(a + 1j * rng.standard_normal(s) if cplx else a)
+
+    L, R, x = rand(13, D, 13), rand(6, D, 6), rand(13, d, d, 6)
+    x[5, -1, -1, 2] = 1e300
+    for W in (np.asfortranarray(rng.standard_normal((D, d, d, D))), rand(D, d, d, D)):
+        out = T.heff_apply(*(Tensor.from_numpy(a) for a in (L, W, W, R, x))).numpy()
+        ref = product_optimal(L, W, W, R, x)
+        assert np.linalg.norm(out / 1e300 - ref / 1e300) <= 1e-13 * np.linalg.norm(ref / 1e300)
+
+
 @pytest.mark.parametrize("prec,cplx", [("f64", False), ("f64", True), ("f32", False)])
 @pytest.mark.parametrize("chi", [(5, 7), (61, 34)])
 def test_mix_profiled_work(ctx, rng, chi, prec, cplx):
