@@ -280,8 +280,13 @@ void small_contract(tnh_ctx *ctx, const Small &s) {
   const int va = (cin || s.I > 32) ? 1 : (i64 || o64) ? 2 : 4;
   p.total = int64_t((s.na + va - 1) / va) * s.nb;
   const int64_t blocks = (p.total + 255) / 256;
-  // split the output columns until the launch has 8 waves per CU
-  const int64_t want = std::max<int64_t>(1, (2 * int64_t(ctx->cu_count) + blocks - 1) / blocks);
+  // Split the output columns towards 8 waves per CU, but not past them: a split reads the input
+  // again. Measured, I = J = 12 / 28, us: FP64 bond 500 (489 blocks) whole 13.7 / 31.6, in two 15.2
+  // / 34.2; 450 (396) 12.9 / 29.2, 14.1 / 31.2; FP32 bond 600 (352) 12.0 / 26.8, 10.7 / 21.7; 450
+  // (199) in two 10.1 / 20.4, in three 11.0 / 21.4; FP64 bond 300 (176) 8.8 / 18.1, 8.4 / 16.1.
+  const int64_t full = 2 * int64_t(ctx->cu_count);
+  int64_t want = std::max<int64_t>(1, (10 * full / blocks + 1) / 10);
+  if (want == 1 && 20 * full >= 29 * blocks) want = 2;  // (one block a CU)
   p.jper = int((s.J + std::min<int64_t>(want, s.J) - 1) / std::min<int64_t>(want, s.J));
   const dim3 grid(unsigned(blocks), unsigned((s.J + p.jper - 1) / p.jper));
   const bool whole = s.I <= 32 && !(cin && cw);
