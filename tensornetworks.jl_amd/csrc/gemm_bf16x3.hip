@@ -51,9 +51,11 @@ __global__ __launch_bounds__(256) void split_bf16_kernel(const T *__restrict__ X
 
 template <typename TC, int BM, int BN>
 void launch_p(hipStream_t s, const Params &p, int batch) {
-  dim3 grid(p.tiles_m * p.tiles_n, batch, p.ksplit);
-  hipLaunchKernelGGL((gemm_kernel<MODE_BF16P, unsigned short, unsigned short, TC, true, false, BM, BN, 1>),
-                     grid, dim3(256), 0, s, p);
+  dim3 grid(p.tiles_m * p.tiles_n, batch);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, p); };
+  if constexpr (std::is_same<TC, float>::value)  // (partial results are FP32)
+    if (p.kper) return go(gemm_kernel<MODE_BF16P, unsigned short, unsigned short, TC, true, false, BM, BN, 1, true>);
+  go(gemm_kernel<MODE_BF16P, unsigned short, unsigned short, TC, true, false, BM, BN, 1>);
 }
 
 }  // namespace

@@ -7,13 +7,19 @@ namespace gk {
 
 template <typename TA, typename TB, typename TC, bool TRA, bool TRB, int BM, int BN>
 static void launch(hipStream_t s, const Params &p, int batch) {
-  dim3 grid(p.tiles_m * p.tiles_n, batch, p.ksplit);
-  if (p.vecA == 1 && p.vecB == 1)
-    hipLaunchKernelGGL((gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 1>), grid, dim3(256), 0, s, p);
+  dim3 grid(p.tiles_m * p.tiles_n, batch);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, p); };
+  const bool aligned = p.vecA == 1 && p.vecB == 1;
+  if constexpr (std::is_same<TC, float>::value)  // (partial results are FP32)
+    if (p.kper)
+      return aligned ? go(gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 1, true>)
+                     : go(gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 2, true>);
+  if (aligned)
+    go(gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 1>);
   else if (p.vecA && p.vecB)
-    hipLaunchKernelGGL((gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 2>), grid, dim3(256), 0, s, p);
+    go(gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 2>);
   else
-    hipLaunchKernelGGL((gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 0>), grid, dim3(256), 0, s, p);
+    go(gemm_kernel<MODE_F32, TA, TB, TC, TRA, TRB, BM, BN, 0>);
 }
 
 template <typename TA, typename TB, typename TC, int BM, int BN>
