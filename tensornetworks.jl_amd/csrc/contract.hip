@@ -31,6 +31,29 @@ struct SmallParams {
   int64_t offJ[kMaxIJ];
 };
 
+// VA consecutive elements at any element address; `left` of them exist when that is fewer. (The
+// type says so: as a plain vector it would promise the compiler an aligned address.)
+template <typename T, int VA>
+struct Run {
+  typedef T V __attribute__((ext_vector_type(VA), aligned(sizeof(T))));
+  __device__ __forceinline__ static V load(const T *q, int left) {
+    if (VA == 1 || left >= VA) return *reinterpret_cast<const V *>(q);
+    V x;
+#pragma unroll
+    for (int u = 0; u < VA; ++u) x[u] = u < left ? q[u] : T(0);
+    return x;
+  }
+  __device__ __forceinline__ static void store(T *q, int left, V x) {
+    if (VA == 1 || left >= VA) {
+      *reinterpret_cast<V *>(q) = x;
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < VA; ++u)
+      if (u < left) q[u] = x[u];
+  }
+};
+
 // out[a, j, b] = sum_i in[a, i, b] * Wc[i, j]; a thread takes VA consecutive a of one b (a
 // fastest, so that a wave's loads and stores are contiguous runs) and jper of the J output
 // columns. NI is I rounded up to a multiple of four (WHOLE), with zeros for the terms past I, so
@@ -52,8 +75,8 @@ __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
   using R = typename std::conditional<std::is_same<TI, double>::value ||
                                           std::is_same<TO, double>::value,
                                       double, float>::type;
-  typedef TI VI __attribute__((ext_vector_type(VA), aligned(sizeof(TI))));
-  typedef TO VO __attribute__((ext_vector_type(VA), aligned(sizeof(TO))));
+  using In = Run<TI, VA>;
+  using Out = Run<TO, VA>;
   extern __shared__ double wsm[];
   R *W = reinterpret_cast<R *>(wsm);
   const int I = p.I, j0 = blockIdx.y * p.jper, nj = min(p.J - j0, p.jper);
@@ -73,32 +96,13 @@ __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
   const int64_t b = idx / nav;
   const TI *in = static_cast<const TI *>(p.in) + a + b * p.sbI;
   TO *out = static_cast<TO *>(p.out) + a + b * p.sbJ;
-  auto load = [&](const auto *q, auto &x) {
-    using V = std::remove_reference_t<decltype(x)>;
-    if (VA == 1 || left >= VA) {
-      x = *reinterpret_cast<const V *>(q);
-    } else {
-#pragma unroll
-      for (int u = 0; u < VA; ++u) x[u] = u < left ? q[u] : 0;
-    }
-  };
-  auto store = [&](auto *q, const auto &x) {
-    using V = std::remove_const_t<std::remove_reference_t<decltype(x)>>;
-    if (VA == 1 || left >= VA) {
-      *reinterpret_cast<V *>(q) = x;
-    } else {
-#pragma unroll
-      for (int u = 0; u < VA; ++u)
-        if (u < left) q[u] = x[u];
-    }
-  };
   R vr[NI][VA], vi[CIN ? NI : 1][VA];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    VI x = 0, y = 0;
+    typename In::V x = 0, y = 0;
     if ((WHOLE && i + 3 < NI) || i < I) {
-      load(in + p.offI[i], x);
-      if constexpr (CIN) load(in + p.in_im + p.offI[i], y);
+      x = In::load(in + p.offI[i], left);
+      if constexpr (CIN) y = In::load(in + p.in_im + p.offI[i], left);
     }
 #pragma unroll
     for (int u = 0; u < VA; ++u) {
@@ -135,24 +139,24 @@ __global__ __launch_bounds__(256) void mix_kernel(SmallParams p) {
       }
     }
     TO *o = out + p.offJ[j0 + j];
-    VO x;
+    typename Out::V x;
     if (p.beta != 0.0) {
-      load(o, x);
+      x = Out::load(o, left);
 #pragma unroll
       for (int u = 0; u < VA; ++u) sr[u] += R(p.beta) * R(x[u]);
       if constexpr (CIN || CW) {
-        load(o + p.out_im, x);
+        x = Out::load(o + p.out_im, left);
 #pragma unroll
         for (int u = 0; u < VA; ++u) si[u] += R(p.beta) * R(x[u]);
       }
     }
 #pragma unroll
     for (int u = 0; u < VA; ++u) x[u] = TO(sr[u]);
-    store(o, x);
+    Out::store(o, left, x);
     if constexpr (CIN || CW) {
 #pragma unroll
       for (int u = 0; u < VA; ++u) x[u] = TO(si[u]);
-      store(o + p.out_im, x);
+      Out::store(o + p.out_im, left, x);
     }
   }
 }
