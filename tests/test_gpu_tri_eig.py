@@ -106,3 +106,29 @@ def test_tri_eig_largest_sides(ctx, rng, cplx, p):
     assert np.abs(got ** 2 - s ** 2).max() <= 1e-13 * np.sqrt(p) * s[0] ** 2
     assert np.abs(u.conj().T @ u - np.eye(p)).max() <= 1e-12
     assert np.linalg.norm((u * got) @ vt - M) <= 1e-12 * np.linalg.norm(M)
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("p,top,solver", [(520, 36, "jacobi"), (520, 40, "tri_eig"), (1601, 194, "jacobi"),
+                                          (1601, 199, "tri_eig")])
+def test_solver_by_active_pairs(ctx, rng, cplx, p, top, solver):
+    """Above side 512 a Gram matrix whose pairs lie mostly below the block Jacobi's floor (only
+    `top` rows of M have weight, top^2 / p^2 of the pairs: 0.0048 and 0.0059 around the line 0.0052
+    at side 520, 0.0147 and 0.0154 around 0.015 at 1601) is solved by it, others by the reduction;
+    both to the same accuracy."""
+    from tnhip import Tensor, ops as T
+
+    w = np.where(np.arange(p) < top, 10.0 ** -(3.0 * np.arange(p) / top), 1e-15)
+    q, _ = np.linalg.qr(randn(rng, (p, p), cplx))
+    M = np.asfortranarray(rng.permutation(w)[:, None] * q)
+    ctx.profile_reset()
+    ctx.profile(True)
+    U, S, Vt, _, fb = T.svd_trunc(Tensor.from_numpy(M), 0.0, 0, 1)
+    ran = {f: int(ctx.profile_read(f)["launches"]) for f in ("jacobi", "tri_eig")}
+    ctx.profile(False)
+    assert ran == {"jacobi": int(solver == "jacobi"), "tri_eig": int(solver == "tri_eig")}
+    assert not fb
+    u, s = U.numpy(), S.numpy()
+    assert np.abs(s ** 2 - w ** 2).max() <= 1e-13 * np.sqrt(p)
+    assert np.abs(u.conj().T @ u - np.eye(p)).max() <= 1e-12
+    assert np.linalg.norm(u @ (u.conj().T @ M) - M) <= 1e-12 * np.linalg.norm(M)
