@@ -434,10 +434,13 @@ Leaves leaves_of(int p) {
     ++g.levels;
     g.leaf = (p + (1 << g.levels) - 1) >> g.levels;
   }
-  // In the range of the one-workgroup solver the blocks are 32, 64, ... wide from position 0, as
-  // its own are: which couplings are torn, and so which small ones deflate, is then the same,
-  // and results agree with it closely (observables after four DMRG passes to 1e-10, against
-  // 3e-9 with equal leaves). Above, equal leaves keep the padding under one per leaf.
+  // Up to side 512 the blocks are 32, 64, ... wide from position 0, as the one-workgroup solver's
+  // are: where T is torn decides which small couplings deflate, and equal leaves lose accuracy on
+  // graded matrices (a gate's tensors against 64-bit LAPACK, blocks of 32 / equal leaves, geometric
+  // mean of 14 seeds: bond 70 3.3e-11 / 1.7e-10, 80 3.3e-11 / 1.2e-10, 150 8.4e-11 / 2.7e-10, 200
+  // 8.8e-11 / 2.3e-10) for 0 - 5% of time (complex side 257 1.52 / 1.47 ms, 160 0.86 / 0.84, 224 1.24 /
+  // 1.25). Above, equal leaves keep the padding under one per leaf; the block Jacobi that had these
+  // sides was further off (bond 300: 1.7e-7, 4.0e-10 here).
   if (g.levels > 0 && p <= dc::kDcPMax) g.leaf = kLeafMax;
   g.Pp = g.leaf << g.levels;
   return g;
@@ -488,29 +491,38 @@ __device__ __forceinline__ bool failed(const DcWork &w) {
   return status == 0;
 }
 
-// One leaf per workgroup, by dc_eig.hpp's tridiagonal solver.
+// One leaf per workgroup, by dc_eig.hpp's tridiagonal solver, which sees its positions of T only:
+// with the padding among them, its deflation threshold would follow that bound on all of T instead
+// of the leaf's own entries, and the small end of a graded matrix, which is where the padding
+// sits, would lose its relative accuracy (a gate's tensors at bond 70, side 140: 2.9e-9 from 64-bit
+// LAPACK with it, 3.4e-11 without).
 __global__ __launch_bounds__(kLeafThreads) void tri_leaf_kernel(DcWork w, double *__restrict__ Q,
                                                                 double *__restrict__ Q2, double *__restrict__ U) {
   __shared__ dc::DcShared sh;
   if (failed(w)) return;
-  const int b = blockIdx.x * w.leaf, s = w.leaf, t = threadIdx.x;
+  const int b = blockIdx.x * w.leaf, s = w.leaf, t = threadIdx.x, r = max(0, min(s, w.p - b));
   const int64_t P = w.Pp, o = b * (P + 1);
-  for (int i = t; i < s; i += kLeafThreads) {
+  for (int e = t; e < s * s; e += kLeafThreads) {
+    const int i = e % s, c = e / s;
+    if (i >= r || c >= r) Q[o + i + c * P] = i == c ? 1.0 : 0.0;
+  }
+  for (int i = r + t; i < s; i += kLeafThreads) w.lam[0][b + i] = w.d[b + i];
+  for (int i = t; i < r; i += kLeafThreads) {
     sh.d[i] = w.d[b + i];
-    sh.e[i] = i + 1 < s ? w.e[b + i] : 0.0;
+    sh.e[i] = i + 1 < r ? w.e[b + i] : 0.0;
   }
   if (t == 0) sh.status = 1;
   __syncthreads();
-  if (s == 1) {
-    if (t == 0) {
+  if (r <= 1) {
+    if (t == 0 && r == 1) {
       Q[o] = 1.0;
       w.lam[0][b] = sh.d[0];
     }
     return;
   }
-  dc::dc_tridiag(dc::DcDeviceEx<kLeafThreads>{}, sh, s, P, Q + o, Q2 + o, U + o);
+  dc::dc_tridiag(dc::DcDeviceEx<kLeafThreads>{}, sh, r, P, Q + o, Q2 + o, U + o);
   __syncthreads();
-  for (int i = t; i < s; i += kLeafThreads) w.lam[0][b + i] = sh.u.c.lam[i];
+  for (int i = t; i < r; i += kLeafThreads) w.lam[0][b + i] = sh.u.c.lam[i];
   if (t == 0 && sh.status == 0) w.info[1] = 0;
 }
 

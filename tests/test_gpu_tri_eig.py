@@ -132,3 +132,21 @@ def test_solver_by_active_pairs(ctx, rng, cplx, p, top, solver):
     assert np.abs(s ** 2 - w ** 2).max() <= 1e-13 * np.sqrt(p)
     assert np.abs(u.conj().T @ u - np.eye(p)).max() <= 1e-12
     assert np.linalg.norm(u @ (u.conj().T @ M) - M) <= 1e-12 * np.linalg.norm(M)
+
+
+@pytest.mark.parametrize("cplx,p", [(True, 44), (True, 76), (True, 140), (False, 109), (False, 140), (False, 220)])
+def test_graded_rows_keep_relative_accuracy(ctx, p, cplx):
+    """M = D B with rows graded over five decades and B random: a solver that starts at the large
+    end resolves each squared singular value relative to itself, to a few eps kappa(B)^2 sqrt(p)
+    (the Gram matrix and the reduction are exact up to eps relative to their rows' and columns'
+    scales). The sides leave the last block of the divide and conquer part padding."""
+    from tnhip import Tensor, ops as T
+
+    rng = np.random.default_rng(p)
+    B = randn(rng, (p, p), cplx)
+    M = np.asfortranarray(B * 10.0 ** np.linspace(0, -5, p)[:, None])
+    _, S, _, _, fb = T.svd_trunc(Tensor.from_numpy(M), 0.0, 0, 1)
+    assert not fb
+    ref = np.linalg.svd(M, compute_uv=False)
+    kappa = np.linalg.cond(B / np.linalg.norm(B, axis=1)[:, None])
+    assert np.abs(S.numpy() / ref - 1).max() <= 16 * 2.3e-16 * np.sqrt(p) * kappa ** 2
