@@ -94,9 +94,15 @@ int tnh_profile_read(tnh_ctx *ctx, const char *family, int64_t *launches, double
  * stream is synchronised once); the fastest is kept for the class if it beats the size
  * rule's tile by at least 3%, else the rule's tile (near-ties stay stable); smaller or
  * batched products, and products issued while the stream is being captured, take the
- * size rule; FP64 products of few tiles run a kernel without tile choices in every mode. mode 0: always the size rule. mode 2: forget the tuned classes. Tiles
- * differ only in the output block a workgroup computes, never in the summation order,
- * so results do not depend on the choice. */
+ * size rule; FP64 products of few tiles run a kernel without tile choices in every mode.
+ * mode 0: always the size rule. mode 2: forget the tuned classes. Tiles differ only in
+ * the output block a workgroup computes, never in the summation order, so results do
+ * not depend on the choice. Apart from tiles, a rule on sizes alone sums some large
+ * products (k from 1024 on) in two to six slices of k, added in FP64. Their partial
+ * results stay in a workspace of the context (2 - 6 M N values, kept until it is
+ * destroyed). A product that is captured, or that finds no memory for them, is summed in
+ * one piece: the same precision, other last bits. tnh_heff_apply does not slice shapes
+ * that tnh_heff_apply_noalloc takes too. */
 int tnh_gemm_autotune(tnh_ctx *ctx, int mode);
 /* The tuned classes as text, one line each: mode, transposes, the timed product's
  * M N K, the chosen and the rule's tile, and the milliseconds of every candidate.

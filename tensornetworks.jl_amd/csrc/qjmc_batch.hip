@@ -708,6 +708,8 @@ __global__ void qb_copy_state_kernel(const double *__restrict__ S, int64_t scap,
 // reduce with the matrix in registers (tri_tail.hpp), which is why a workgroup has 512 threads.
 // Measured on 64 trajectories x 16 steps, N = 16, bonds growing to 45: a launch 10.1 -> 5.9 ms
 // (register reduction 8.3, then products 16 k at a time and kept columns in one round).
+// Larger sides reduce in LDS and L2 on these 512 threads (they had 1024); with the other two changes
+// whole runs at N = 16 take, before -> now: sides to 128 801 -> 524 ms, 256 1310 -> 833, 504 2711 -> 1800.
 
 constexpr int WT = 512;  // threads per trajectory workgroup: 256 registers each
 constexpr int WW = WT / 64;         // waves

@@ -1,11 +1,12 @@
-// Eigen-decomposition of a Hermitian matrix (sides: tri_eig.hpp) spread over the whole GPU: Householder reduction to a real symmetric tridiagonal matrix, divide and conquer with
-// one launch per phase and level, back-transformation by blocked reflectors on the matrix
-// cores. It replaces two solvers for the Gram matrices of cold splits: the one-workgroup
-// reduction (whose p steps stream the matrix through one CU: 25 ms at p = 512) and, above
-// 512, the block Jacobi (17-20 sweeps over the matrix).
+// Eigen-decomposition of a Hermitian matrix (sides: tri_eig.hpp) spread over the whole GPU:
+// Householder reduction to a real symmetric tridiagonal matrix, divide and conquer with one
+// launch per phase and level, back-transformation by blocked reflectors on the matrix cores. It
+// replaces two solvers for the Gram matrices of splits: the one-workgroup reduction (whose p
+// steps stream the matrix through one CU: 25 ms at p = 512) and, above 512 for matrices that are
+// not mostly below its noise floor (svd.hip), the block Jacobi (17-20 sweeps over the matrix).
 //
 // Measured (graded Gram matrices, MI355X; before -> now, eigensolver only): real 160 1.9 ->
-// 0.66 ms, 512 30 -> 2.6 ms, 602 22 -> 3.1 ms, 4096 470 -> 102 ms; complex 160 2.6 -> 0.87
+// 0.64 ms, 512 30 -> 2.5 ms, 602 22 -> 3.1 ms, 4096 470 -> 102 ms; complex 160 2.6 -> 0.86
 // ms, 512 51 -> 3.7 ms. The kept vectors' error against 64-bit LAPACK falls with it (4096,
 // weights down to 1e-3 of the largest: 2.6e-7 -> 2.8e-11), since a reduction that starts at
 // the large end of a graded matrix keeps its small eigenvalues' relative accuracy.
@@ -14,7 +15,7 @@
 // column (tri_col_kernel): every workgroup repeats the O(n) part of the step (the pending
 // rank-2 update of the pivot column, its reflector), then updates its own columns and forms
 // their entries of y = A v. The launch boundary is the only grid-wide synchronisation. The
-// last kTailMax columns run in one workgroup with the active matrix in registers
+// last tail_max columns run in one workgroup with the active matrix in registers
 // (tri_tail_kernel), two barriers per column.
 //
 // Divide and conquer. Leaves of at most 32 are solved by dc_eig.hpp's tridiagonal solver, one
